@@ -131,6 +131,16 @@ __host__ __device__ __forceinline__ int round_near(float x, float& k) {
 #endif
 }
 
+// T_k - T for the grid point k.  In float the step is taken in two parts: its
+// FP32 value is 1.5e-8 too large, and T_k with it, so every integral would
+// lean the same way (F_6 8e-8 on average over T < 30, now 5e-10), which a sum
+// of millions of them does not average out.
+__host__ __device__ __forceinline__ double grid_offset(double k, double T) { return k * kBoysStep - T; }
+__host__ __device__ __forceinline__ float grid_offset(float k, float T) {
+  constexpr float hi = (float)kBoysStep, lo = (float)(kBoysStep - (double)hi);
+  return fmaf(k, lo, fmaf(k, hi, -T));
+}
+
 // 1/sqrt(s) for s > 0: the hardware estimate refined by two Newton steps
 // y <- y (3/2 - s/2 y^2), each of which squares the relative error.
 __host__ __device__ __forceinline__ double rsqrt_nr(double s) {
@@ -169,7 +179,7 @@ __host__ __device__ __forceinline__ void boys(R T, R (&F)[L + 1], const double* 
   if (T < R(kBoysTCut[L] - 0.5 * kBoysStep)) {
     R kr;
     const int k = round_near(T * R(1.0 / kBoysStep), kr);
-    const R d = kr * R(kBoysStep) - T;  // expansion in (T_k - T)
+    const R d = grid_offset(kr, T);  // expansion in (T_k - T)
     const double* row = lds + k * kBoysLdsW;
     // F_L(T) = sum_j F_{L+j}(T_k) (T_k - T)^j / j!
     R s = R(row[NT - 1]);
