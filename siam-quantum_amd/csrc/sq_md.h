@@ -131,14 +131,31 @@ __host__ __device__ __forceinline__ int round_near(float x, float& k) {
 #endif
 }
 
-// T_k - T for the grid point k.  In float the step is taken in two parts: its
-// FP32 value is 1.5e-8 too large, and T_k with it, so every integral would
-// lean the same way (F_6 8e-8 on average over T < 30, now 5e-10), which a sum
-// of millions of them does not average out.
+// In an FP32 evaluation the rounding of a constant leans the same way in every
+// integral, and a J element sums millions of them, so constants enter with a
+// second FP32 part there: 0.1 of the table step is 1.5e-8 too large, 1/3, 1/5
+// and 1/7 of the recursion 3e-8, 1.5e-8 and 4e-8, which left F_0 at L = 6
+// 1.2e-7 too large on average over T < 30 (now 7e-10).
+// T_k - T for the grid point k:
 __host__ __device__ __forceinline__ double grid_offset(double k, double T) { return k * kBoysStep - T; }
 __host__ __device__ __forceinline__ float grid_offset(float k, float T) {
   constexpr float hi = (float)kBoysStep, lo = (float)(kBoysStep - (double)hi);
   return fmaf(k, lo, fmaf(k, hi, -T));
+}
+// x / (2 M + 1):
+template <int M>
+__host__ __device__ __forceinline__ double div_odd(double x) { return x * (1.0 / (2 * M + 1)); }
+template <int M>
+__host__ __device__ __forceinline__ float div_odd(float x) {
+  constexpr float hi = (float)(1.0 / (2 * M + 1)), lo = (float)(1.0 / (2 * M + 1) - (double)hi);
+  return M == 0 ? x : fmaf(x, hi, x * lo);
+}
+// x sqrt(pi) / 2:
+constexpr double kHalfSqrtPi = 0.88622692545275801365;
+__host__ __device__ __forceinline__ double mul_half_sqrt_pi(double x) { return kHalfSqrtPi * x; }
+__host__ __device__ __forceinline__ float mul_half_sqrt_pi(float x) {
+  constexpr float hi = (float)kHalfSqrtPi, lo = (float)(kHalfSqrtPi - (double)hi);
+  return fmaf(x, hi, x * lo);
 }
 
 // 1/sqrt(s) for s > 0: the hardware estimate refined by two Newton steps
@@ -198,13 +215,13 @@ __host__ __device__ __forceinline__ void boys(R T, R (&F)[L + 1], const double* 
       const R e = R(row[kBoysTaylor]) * x, t2 = T + T;
       sfor<L>([&](auto mm) {
         constexpr int m = L - 1 - decltype(mm)::value;
-        F[m] = (t2 * F[m + 1] + e) * R(1.0 / (2 * m + 1));
+        F[m] = div_odd<m>(t2 * F[m + 1] + e);
       });
     }
   } else {
     // large T: F_0 = sqrt(pi/T)/2, F_{m+1} = (2m+1) F_m / (2T)
     const R y = rsqrt_nr(T);
-    F[0] = R(0.88622692545275801365) * y;
+    F[0] = mul_half_sqrt_pi(y);
     if constexpr (L > 0) {
       const R h = R(0.5) * y * y;
       sfor<L>([&](auto mm) {
@@ -297,16 +314,18 @@ struct RPlan {
 };
 
 // pref R^{(0)}_{tuv} for t+u+v <= L, built level by level from
-// R^{(n)}_{000} = (-2 alpha)^n F_n.
+// R^{(n)}_{000} = (-2 alpha)^n F_n.  alpha and its powers are FP64 in an FP32
+// evaluation too: alpha is the same for all quartets of a kind, so its
+// rounding would lean the same way in all of them.
 template <int L, typename Rl = double>
 __host__ __device__ __forceinline__ void herm_R(Rl (&R)[nherm(L)], const Rl (&F)[L + 1],
-                                       Rl alpha, Rl X, Rl Y, Rl Z, Rl pref = Rl(1)) {
+                                       double alpha, Rl X, Rl Y, Rl Z, double pref = 1.0) {
   constexpr RPlan<L> plan{};
   Rl lev[L + 1][nherm(L)];
-  Rl m2a = Rl(-2) * alpha, pw = pref;
+  double m2a = -2.0 * alpha, pw = pref;
   sfor<L + 1>([&](auto nn) {
     constexpr int n = decltype(nn)::value;
-    lev[n][0] = pw * F[n];
+    lev[n][0] = Rl(pw) * F[n];
     pw *= m2a;
   });
   // level n holds orders up to L-n; build from n = L-1 down to 0

@@ -28,3 +28,17 @@ def test_fp32_boys_unbiased(L):
     mean = ((F[:, L] - ref) / ref).mean()
     print(f"L={L}: mean relative error {mean:.2e}", flush=True)
     assert abs(mean) < 2.0 ** -26
+
+
+@pytest.mark.parametrize("L", list(range(1, 10)))
+def test_fp32_boys_recursion_unbiased(L):
+    T = np.random.default_rng(60 + L).uniform(0.1, 30.0, 40000).astype(np.float32).astype(np.float64)
+    F = np.zeros((len(T), L + 1))
+    lib().sqjk_boys.argtypes = [C.c_int, C.c_int, C.POINTER(C.c_double), C.c_int, C.c_int, C.POINTER(C.c_double)]
+    assert lib().sqjk_boys(L, len(T), dptr(T), 1, 0, dptr(F)) == 0, lib().sqjk_errmsg()
+    mean = []
+    for m in range(L):
+        ref = gammainc(m + 0.5, T) * gamma(m + 0.5) / (2 * T ** (m + 0.5))
+        mean.append(((F[:, m] - ref) / ref).mean())
+    print(f"L={L}: mean relative errors " + " ".join(f"{x:.1e}" for x in mean), flush=True)
+    assert max(abs(x) for x in mean) < 2.0 ** -26
