@@ -46,6 +46,13 @@ typedef struct {
 	int launches;          /* kernel launches in this build                */
 } sqjk_stats;
 
+/* Frees the device and pinned host blocks that the library keeps for the next
+ * context (4 GiB at most, and up to an eighth of the device beside them while
+ * a context that has run MP2 is alive) and returns their bytes: for a program
+ * that needs the memory elsewhere.  The library's own allocations do this by
+ * themselves when they fail.  No counterpart in the reference. */
+long long sqjk_release_cached(void);
+
 /* Create a context for one basis.  schwarz_basis: optional n x n matrix of
  * sqrt|(pq|pq)| (as from create_Schwarz); NULL computes it on the device.
  * device: HIP device ordinal.  Returns SQJK_OK and *out on success. */

@@ -13,6 +13,8 @@ double sqjk_dropin_mixed_internal();
 // would wait for the whole device)
 void* sq_device_block(size_t bytes);
 void sq_device_release(void* p);
+// bytes the cache holds of the current device (free to a request that needs them)
+size_t sq_device_cached();
 
 // MP2 energy from the dense AO pair matrix *dV (sq_mp2.hip): one spin block
 // (closed shell) or two (alpha, beta: same-spin and opposite-spin terms).

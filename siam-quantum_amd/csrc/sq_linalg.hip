@@ -21,9 +21,11 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/sq_scf.h"
+#include "sq_internal.h"
 #include "sq_linalg_dev.h"
 
 namespace {
@@ -146,17 +148,20 @@ int ensure(Work& w, int n, hipStream_t st) {
   if (w.n >= n) return 0;
   if (w.A) {
     (void)hipStreamSynchronize(w.st);
-    (void)hipFree(w.A); (void)hipFree(w.B); (void)hipFree(w.W); (void)hipFree(w.E);
-    (void)hipFree(w.P); (void)hipFree(w.X); (void)hipFree(w.info); (void)hipFree(w.red);
+    void* p[] = {w.A, w.B, w.P, w.X, w.W, w.E, w.red, w.info};
+    for (void* q : p) sq_device_release(q);
     w.A = w.B = w.W = w.E = w.P = w.X = w.red = nullptr;
     w.info = nullptr;
   }
   w.metric_n = 0;
   const size_t nn = (size_t)n * n;
-  if (hipMalloc(&w.A, nn * 8) != hipSuccess || hipMalloc(&w.B, nn * 8) != hipSuccess ||
-      hipMalloc(&w.P, nn * 8) != hipSuccess || hipMalloc(&w.X, nn * 8) != hipSuccess ||
-      hipMalloc(&w.W, (size_t)n * 8) != hipSuccess || hipMalloc(&w.E, (size_t)n * 8) != hipSuccess ||
-      hipMalloc(&w.info, sizeof(rocblas_int)) != hipSuccess || hipMalloc(&w.red, 4 * sizeof(double)) != hipSuccess) {
+  auto get = [](auto** p, size_t bytes) {
+    *p = static_cast<std::remove_pointer_t<decltype(p)>>(sq_device_block(bytes));
+    return *p != nullptr;
+  };
+  if (!get(&w.A, nn * 8) || !get(&w.B, nn * 8) || !get(&w.P, nn * 8) || !get(&w.X, nn * 8) ||
+      !get(&w.W, (size_t)n * 8) || !get(&w.E, (size_t)n * 8) || !get(&w.info, sizeof(rocblas_int)) ||
+      !get(&w.red, 4 * sizeof(double))) {
     w.n = 0;
     return -1;
   }
@@ -167,8 +172,7 @@ int ensure(Work& w, int n, hipStream_t st) {
 void release(Work& w) {
   if (w.st) (void)hipStreamSynchronize(w.st);
   void* p[] = {w.A, w.B, w.P, w.X, w.W, w.E, w.red, w.info};
-  for (void* q : p)
-    if (q) (void)hipFree(q);
+  for (void* q : p) sq_device_release(q);
   if (w.h) (void)rocblas_destroy_handle(w.h);
   if (w.own_stream && w.st) (void)hipStreamDestroy(w.st);
   w = Work{};

@@ -212,6 +212,7 @@ int first_half(Ctx& c, const double* dV, const SqMp2Spin& sp, Half& H) {
   const double one = 1.0, zero = 0.0;
   size_t freeb = 0, totb = 0;
   if (hipMemGetInfo(&freeb, &totb) != hipSuccess) return c.bad("hipMemGetInfo failed");
+  freeb += sq_device_cached();
   const size_t blk = H.blk = std::min<size_t>(pair_block(npr, (size_t)n * n * 8 + (size_t)nc * n * 8, freeb),
                                               (size_t)INT32_MAX / std::max(nc, nv));
   double *dVf = nullptr, *dT = nullptr;
@@ -243,6 +244,7 @@ int second_half(Ctx& c, const Half& H, const SqMp2Spin& bra, const SqMp2Spin& ke
   const double one = 1.0, zero = 0.0;
   size_t freeb = 0, totb = 0;
   if (hipMemGetInfo(&freeb, &totb) != hipSuccess) return c.bad("hipMemGetInfo failed");
+  freeb += sq_device_cached();
   const size_t per_x = ((size_t)n * n + (size_t)n * ket.nc + (size_t)ket.nc * ket.nv) * 8;
   const size_t most = std::min<size_t>(std::min<size_t>(freeb / 2, (size_t)2 << 30) / per_x,
                                        (size_t)INT32_MAX / std::max(ket.nc, 1));

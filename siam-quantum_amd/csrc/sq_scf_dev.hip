@@ -268,8 +268,7 @@ int alloc_mats(sqscf_ctx* c, int n) {
     for (int k = 0; k < 2; ++k)
       if (!get(&c->hp[s][k], nn * 8) || !get(&c->he[s][k], nn * 8))
         return scf_fail(SQJK_ENOMEM, "SCF device allocation failed");
-  if (!c->partial && (hipMalloc(&c->partial, kRedBlocks * kMaxSums * 8) != hipSuccess ||
-                      hipMalloc(&c->sums, kMaxSums * 8) != hipSuccess))
+  if (!c->partial && (!get(&c->partial, kRedBlocks * kMaxSums * 8) || !get(&c->sums, kMaxSums * 8)))
     return scf_fail(SQJK_ENOMEM, "SCF device allocation failed");
   c->cap = n;
   return SQJK_OK;
@@ -637,8 +636,8 @@ void sqscf_destroy(sqscf_ctx* c) {
   if (c->st) (void)hipStreamSynchronize(c->st);
   sqla::release(c->lw);
   free_mats(c);
-  if (c->partial) (void)hipFree(c->partial);
-  if (c->sums) (void)hipFree(c->sums);
+  sq_device_release(c->partial);
+  sq_device_release(c->sums);
   if (c->jk) sqjk_destroy(c->jk);
   delete c;
 }

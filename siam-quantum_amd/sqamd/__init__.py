@@ -5,4 +5,4 @@ raises if the library is not built: there is no Python or CPU fallback.
 """
 from .abi import (Basis, GTOBasis, GTOBasisSet, Mol, Molecule, Option,  # noqa: F401
                   basis_from_ptr, default_option, dptr)
-from .engine import JKEngine, lib, library_path  # noqa: F401
+from .engine import JKEngine, lib, library_path, release_cached  # noqa: F401

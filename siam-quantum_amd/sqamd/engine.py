@@ -66,6 +66,13 @@ def _check(rc, what):
         raise RuntimeError(f"{what} failed ({rc}): {lib().sqjk_errmsg().decode()}")
 
 
+def release_cached():
+    """Frees the device and pinned blocks the library keeps for its next
+    context (sqjk_release_cached); returns their bytes."""
+    lib().sqjk_release_cached.restype = C.c_longlong
+    return lib().sqjk_release_cached()
+
+
 class JKEngine:
     """One molecule's J/K context on the device (sqjk_create/sqjk_build)."""
 

@@ -2,7 +2,9 @@
 refuses requests beyond its size and remembers the error of a refused one,
 like the HIP runtime.  Each case is a few lines of C++; a failed CHECK prints
 its line."""
+import glob
 import os
+import re
 import subprocess
 
 import pytest
@@ -99,3 +101,78 @@ def test_smallest_fitting_block(tmp_path):
   CHECK(c.get(200, false) == a);
   c.put(nullptr);
 """)
+
+
+def test_large_blocks_follow_their_user(tmp_path):
+    """Device blocks above 256 MiB: 4 GiB without a large user, an eighth of
+    the device beside that with one, nothing of it after it."""
+    _run(tmp_path, """
+  auto pass = [&](size_t big) {
+    void* a = c.get(big, false); void* b = c.get(5 * G, false); void* s = c.get(100, false);
+    c.put(a); c.put(b); c.put(s);
+  };
+  pass(17 * G);
+  CHECK(c.cached(0) == 100);
+  c.large_user(1);
+  pass(17 * G);
+  CHECK(c.cached(0) == 22 * G + 100);
+  const int n = st.mallocs;
+  pass(17 * G);
+  CHECK(st.mallocs == n);  // all of them were there
+  c.put(c.get(15 * G, false));  // takes the 17 GiB block and gives it back
+  CHECK(c.cached(0) == 22 * G + 100);
+  void* x = c.get(30 * G, false);
+  c.put(x);  // 52 GiB would pass the eighth
+  CHECK(c.cached(0) == 22 * G + 100);
+  c.large_user(1); c.large_user(-1);
+  CHECK(c.cached(0) == 22 * G + 100);
+  c.large_user(-1);
+  CHECK(c.cached(0) == 100);
+  CHECK(c.trim() == 100 && c.cached(0) == 0 && st.used[0] == 0);
+""")
+
+
+def test_large_blocks_leave_half_the_device(tmp_path):
+    """With less than half of the device free, by whomever, only the 4 GiB."""
+    _run(tmp_path, """
+  c.large_user(1);
+  st.used[0] = 130 * G;  // another process, or another allocator of this one
+  void* a = c.get(10 * G, false); void* b = c.get(10 * G, false);
+  c.put(a);  // 138 GiB free
+  CHECK(c.cached(0) == 0);
+  c.put(b);  // 148 GiB free with a gone
+  CHECK(c.cached(0) == 10 * G);
+  a = c.get(10 * G, false);
+  CHECK(a == b);
+  st.used[0] += 10 * G;
+  c.put(a);
+  CHECK(c.cached(0) == 0);
+""")
+
+
+def test_pinned_and_devices_apart(tmp_path):
+    """Pinned memory never passes 4 GiB, and each device has its own eighth."""
+    _run(tmp_path, """
+  c.large_user(1);
+  void* h = c.get(5 * G, true); void* g = c.get(3 * G, true);
+  c.put(h); c.put(g);
+  CHECK(st.pinned == 3 * G);
+  void* a = c.get(30 * G, false);
+  c.put(a);
+  st.dev = 1;
+  void* b = c.get(30 * G, false);
+  c.put(b);
+  CHECK(c.cached(0) == 30 * G && c.cached(1) == 30 * G);
+  CHECK(c.get(20 * G, false) == b);
+  st.dev = 0;
+  c.put(b);  // of the other device: not beyond the 4 GiB
+  CHECK(c.cached(1) == 0 && st.used[1] == 0);
+""")
+
+
+def test_device_memory_in_one_place():
+    """Every allocation of the library goes through the cache, which gives up
+    its blocks when the device is full: no other source calls the runtime's."""
+    calls = [(os.path.basename(f), line.strip()) for f in sorted(glob.glob(os.path.join(CSRC, "*")))
+             for line in open(f) if re.search(r"\bhip(Host)?Malloc(Async)?\(", line.split("//")[0])]
+    assert len(calls) == 1 and calls[0][0] == "sq_jk_engine.hip", calls
