@@ -164,6 +164,13 @@ int sqjk_class_work(sqjk_ctx *ctx, long long *quartets, long long *prim_quartets
 int sqjk_set_tuning(sqjk_ctx *ctx, const int *rows, const int *split_budget, const int *grid_over);
 int sqjk_get_tuning(const sqjk_ctx *ctx, int *rows, int *split_budget, int *grid_over);
 
+/* Tiles of the context's present work plan: those of the J/K build, those of
+ * one wavefront (gradient, integral store, work count; each kind is made by
+ * the first call that reads it, 0 until then), and the bra rows of the longest
+ * build tile of every class pair (6 x 6).  Any pointer may be NULL.
+ * No counterpart in the reference (measurement support). */
+int sqjk_plan_tiles(const sqjk_ctx *ctx, long long *build_tiles, long long *wave_tiles, int *longest);
+
 /* ---- batches: many molecules' J/K builds as one set of launches ----
  * A batch joins existing contexts (which must outlive it; their geometry
  * must not change while it exists).  Per (class pair, precision, spin mode)

@@ -140,6 +140,16 @@ class JKEngine:
         lq = [c[0] for c in self.class_stats()]
         return [(lq[i], q[i], p[i], q32[i], p32[i]) for i in range(k)]
 
+    def plan_tiles(self):
+        """Tiles of the present work plan (sqjk_plan_tiles): build tiles, wavefront
+        tiles, rows of the longest build tile per class pair (6 x 6)."""
+        b, w, r = C.c_longlong(), C.c_longlong(), np.zeros((6, 6), dtype=np.int32)
+        L = lib()
+        L.sqjk_plan_tiles.argtypes = [C.c_void_p, C.POINTER(C.c_longlong), C.POINTER(C.c_longlong), C.POINTER(C.c_int)]
+        _check(L.sqjk_plan_tiles(self._h, C.byref(b), C.byref(w), r.ctypes.data_as(C.POINTER(C.c_int))),
+               "sqjk_plan_tiles")
+        return b.value, w.value, r
+
     def set_profile(self, on=True):
         _check(lib().sqjk_set_profile(self._h, int(on)), "sqjk_set_profile")
 
