@@ -154,7 +154,11 @@ int sqjk_class_work(sqjk_ctx *ctx, long long *quartets, long long *prim_quartets
 /* Work-plan tuning per class pair (arrays of 6 x 6 ints indexed
  * [bra pair class][ket pair class], pair classes ss, ps, pp, ds, dp, dd; any
  * may be NULL to keep the current values; all NULL restores the defaults):
- *   rows          bra rows per tile (1..64),
+ *   rows          bra rows per tile (1..64); for the classes whose tiles a
+ *                 workgroup shares, rows per wavefront of it (4 or 8 of them,
+ *                 64 rows a tile at most).  A table other than the default one
+ *                 holds for the tiles of the gradient and the integral store
+ *                 too, one wavefront each,
  *   split_budget  integral-primitive products per lane and tile above which
  *                 a segment's ket primitive pairs are split over tiles,
  *   grid_over     workgroups per launch as a multiple of those the device
