@@ -52,7 +52,7 @@ def test_covers_every_buffer(make, uhf):
     for X, (la, lb) in enumerate(CLASS):
         need += npair[X] * (40 + 8 * ncart(la) * ncart(lb))                        # pairs, J by pair
         need += npair[X] * n * (ncart(la) + ncart(lb)) * 8 * (2 if uhf else 1)     # exchange staging
-        need += nprim[X] * (64 + _table_stride(la, lb) * 8)                        # primitives, bra tables
+        need += nprim[X] * (64 + _table_stride(la, lb) * (8 + 4))                  # primitives, FP64 and FP32 bra tables
     L = lib()
     L.sqjk_footprint_bytes.restype = C.c_longlong
     got = L.sqjk_footprint_bytes(n, bas.ptr, int(uhf), 0)
