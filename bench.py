@@ -215,6 +215,15 @@ def scf_solves(name, nsolve, mixed_thr):
     return out
 
 
+def kernel_name(lq):
+    """Kernel of the closed-shell FP64 build for the class, as a profiler names it."""
+    if tuple(lq) == (2, 2, 2, 2):
+        return "k_class_wave<2, 2, 2, 2, 0, double>" if os.environ.get("SQJK_DD_KERNEL") == "wave" \
+            else "k_class_wd<2, 2, 2, 2, 0>"
+    from sqamd import workmodel
+    return "k_class<%d, %d, %d, %d, 0, double, %d>" % (*lq, workmodel.class_block(*lq))
+
+
 def profile_traffic(kernel):
     """HBM-side bytes of `kernel` per build (all of its launches in one
     build) from the committed rocprofv3 counter summary (FETCH_SIZE and
@@ -441,11 +450,7 @@ def main():
               for lq, wq, wp, _, _ in work]
     dom = int(np.argmax(cls_ms))
     dlq = work[dom][0]
-    if dlq == (2, 2, 2, 2):
-        dname = "k_class_wave<2, 2, 2, 2, 0, double>" if os.environ.get("SQJK_DD_KERNEL") == "wave" \
-            else "k_class_wd<2, 2, 2, 2, 0>"
-    else:
-        dname = "k_class<%d, %d, %d, %d, 0, double, %d>" % (dlq + (512 if workmodel.class_block(*dlq) == 512 else 256,))
+    dname = kernel_name(dlq)
     dach = cflops[dom] / (cls_ms[dom] / 1e3) / 1e12
     build_ach = sum(cflops) / (kernel_ms / 1e3) / 1e12
     traffic, traffic_src = profile_traffic(dname)
