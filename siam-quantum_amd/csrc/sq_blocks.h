@@ -37,6 +37,7 @@ class BlockCache {
     if (best < kept.size()) {
       const Block b = kept[best];
       kept.erase(kept.begin() + (long)best);
+      if (!b.large) small_bytes -= b.bytes;
       live.push_back(b);
       return b.p;
     }
@@ -61,10 +62,12 @@ class BlockCache {
         Block b = live[i];
         live.erase(live.begin() + (long)i);
         b.large = keep_large_locked(b);
-        if (b.large || bytes_locked([](const Block& k) { return !k.large; }) + b.bytes <= kMost)
+        if (b.large || small_bytes + b.bytes <= kMost) {
           kept.push_back(b);
-        else
+          if (!b.large) small_bytes += b.bytes;
+        } else {
           (void)mem.free(b.p, b.host);
+        }
         return;
       }
   }
@@ -119,6 +122,7 @@ class BlockCache {
     const size_t n = bytes_locked([](const Block&) { return true; });
     for (const Block& b : kept) (void)mem.free(b.p, b.host);
     kept.clear();
+    small_bytes = 0;
     return n;
   }
 
@@ -126,5 +130,6 @@ class BlockCache {
   std::mutex mu;
   std::vector<Block> kept;  // cached, free
   std::vector<Block> live;  // handed out
+  size_t small_bytes = 0;   // of the kept blocks that are not large
   int users = 0;
 };
