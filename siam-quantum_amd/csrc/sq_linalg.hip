@@ -2,10 +2,10 @@
 //
 // Generalised symmetric eigenproblem F C = S C e on the device, behind the
 // reference's src/lin.h surface, and the same operations on device-resident
-// matrices for the SCF that stays on the device (sqla:: in sq_linalg_dev.h).  S is fixed during an SCF, so its Cholesky
-// factor S = U^T U and X = U^-1 are computed once per metric (rocSOLVER
-// dpotrf/dtrtri) and every solve is X^T F X (two DGEMMs), rocSOLVER dsyevd
-// and C = X C' (one DGEMM):
+// matrices for the SCF that stays on the device (sqla:: in sq_linalg_dev.h).
+// S is fixed during an SCF, so its Cholesky factor S = U^T U and X = U^-1 are
+// computed once per metric (blocked, set_metric below) and every solve is
+// X^T F X (two DGEMMs), rocSOLVER dsyevd and C = X C' (one DGEMM):
 //   gen_sym_eigen      <- src/lin.h:20 (src/lin.c:66-177, LAPACK dspgvd)
 //   gen_sym_SomeEigen  <- src/lin.h:24 (src/lin.c:195-307, LAPACK dspgvx)
 //   linear_solver      <- src/lin.h:30 (src/lin.c:320-391, LAPACK dgesv)
@@ -30,12 +30,60 @@
 
 namespace {
 
-// strictly lower triangle (column-major) set to zero
-__global__ void k_zero_lower(double* X, int n) {
-  const size_t nn = (size_t)n * n;
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < nn; e += (size_t)gridDim.x * blockDim.x) {
-    const int j = (int)(e / n), i = (int)(e - (size_t)j * n);
-    if (i > j) X[e] = 0.0;
+__global__ void k_zero(double* X, size_t nn) {
+  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < nn; e += (size_t)gridDim.x * blockDim.x) X[e] = 0.0;
+}
+
+// One workgroup: the diagonal block A (m x m, m <= kNB, column-major with
+// leading dimension n, upper triangle read) = U^T U, and V = U^-1 (upper
+// triangle written, leading dimension n).  k0: the block's first row in the
+// whole matrix.  *info: the first minor that is not positive definite (from
+// 1), set to 0 by the first block; the rest of a matrix without a factor is
+// worked through with a unit pivot.
+// Bound by its m steps of two barriers.
+constexpr int kNB = 64, kDiagBlock = 256, kDiagLd = kNB + 1;
+constexpr size_t kDiagLds = sizeof(double) * 2 * kNB * kDiagLd;
+__global__ void __launch_bounds__(kDiagBlock) k_chol_diag(const double* __restrict__ A, double* __restrict__ V, int m,
+                                                          int n, int k0, rocblas_int* info) {
+  extern __shared__ double chol_lds[];
+  double *u = chol_lds, *v = chol_lds + kNB * kDiagLd;  // [row][column]
+  for (int e = threadIdx.x; e < m * m; e += kDiagBlock) {
+    const int i = e % m, j = e / m;
+    u[i * kDiagLd + j] = i <= j ? A[(size_t)j * n + i] : 0.0;
+    v[i * kDiagLd + j] = 0.0;
+  }
+  if (threadIdx.x == 0 && k0 == 0) *info = 0;
+  __syncthreads();
+  for (int c = 0; c < m; ++c) {
+    double d = u[c * kDiagLd + c];
+    const bool ok = d > 0.0;  // not for a NaN either
+    if (!ok) d = 1.0;
+    const double r = 1.0 / sqrt(d);
+    __syncthreads();  // all have read the pivot
+    if (threadIdx.x == 0 && !ok && *info == 0) *info = k0 + c + 1;
+    for (int j = c + threadIdx.x; j < m; j += kDiagBlock)
+      u[c * kDiagLd + j] = j == c ? sqrt(d) : u[c * kDiagLd + j] * r;
+    __syncthreads();
+    const int w = m - c - 1;
+    for (int e = threadIdx.x; e < w * w; e += kDiagBlock) {
+      const int i = c + 1 + e / w, j = c + 1 + e % w;
+      if (j >= i) u[i * kDiagLd + j] -= u[c * kDiagLd + i] * u[c * kDiagLd + j];
+    }
+    __syncthreads();
+  }
+  // column j of V by back substitution, a thread each
+  if ((int)threadIdx.x < m) {
+    const int j = threadIdx.x;
+    for (int i = j; i >= 0; --i) {
+      double t = i == j ? 1.0 : 0.0;
+      for (int k = i + 1; k <= j; ++k) t -= u[i * kDiagLd + k] * v[k * kDiagLd + j];
+      v[i * kDiagLd + j] = t / u[i * kDiagLd + i];
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < m * m; e += kDiagBlock) {
+    const int i = e % m, j = e / m;
+    V[(size_t)j * n + i] = v[i * kDiagLd + j];
   }
 }
 
@@ -189,18 +237,42 @@ const char* what(const Work& w, int rc) {
   return buf;
 }
 
+// Right-looking Cholesky by blocks of kNB columns and the inverse of the
+// factor, block column by block column.  rocSOLVER's dpotrf, used here
+// before, has left a row of the factor wrong once in a few hundred calls with
+// other streams at work on the device (never alone).
 int set_metric(Work& w, int n, const double* dS) {
   const size_t nn = (size_t)n * n;
   w.metric_n = 0;
-  if ((w.last_hip = hipMemcpyAsync(w.X, dS, nn * 8, hipMemcpyDeviceToDevice, w.st)) != hipSuccess) return -3;
-  if (rocsolver_dpotrf(w.h, rocblas_fill_upper, n, w.X, n, w.info) != rocblas_status_success) return -4;
+  // A: the trailing matrix; P: the blocks of U right of the diagonal; X: V of
+  // every diagonal block, then the blocks above them; B: a block column
+  if ((w.last_hip = hipMemcpyAsync(w.A, dS, nn * 8, hipMemcpyDeviceToDevice, w.st)) != hipSuccess) return -3;
+  hipLaunchKernelGGL(k_zero, dim3(grid_nn(nn)), dim3(256), 0, w.st, w.X, nn);
+  const rocblas_operation N = rocblas_operation_none, T = rocblas_operation_transpose;
+  auto mm = [&](rocblas_operation ta, int m, int k, int c, double alpha, const double* a, const double* b, double beta,
+                double* d) {
+    return rocblas_dgemm(w.h, ta, N, m, c, k, &alpha, a, n, b, n, &beta, d, n) == rocblas_status_success;
+  };
+  auto at = [&](double* M, int i, int j) { return M + (size_t)j * n + i; };
+  for (int k = 0; k < n; k += kNB) {
+    const int m = std::min(kNB, n - k), r = n - k - m;
+    hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(kDiagBlock), kDiagLds, w.st, at(w.A, k, k), at(w.X, k, k), m, n, k,
+                       w.info);
+    if (hipGetLastError() != hipSuccess) return -3;
+    if (r == 0) break;
+    // U(k, rest) = V^T A(k, rest); A(rest, rest) -= U(k, rest)^T U(k, rest)
+    if (!mm(T, m, m, r, 1.0, at(w.X, k, k), at(w.A, k, k + m), 0.0, at(w.P, k, k + m)) ||
+        !mm(T, r, m, r, -1.0, at(w.P, k, k + m), at(w.P, k, k + m), 1.0, at(w.A, k + m, k + m)))
+      return -4;
+  }
+  // X(above, j) = -X(above, above) U(above, j) V_j
+  for (int j = kNB; j < n; j += kNB) {
+    const int m = std::min(kNB, n - j);
+    if (!mm(N, j, m, m, 1.0, at(w.P, 0, j), at(w.X, j, j), 0.0, w.B) ||
+        !mm(N, j, j, m, -1.0, w.X, w.B, 0.0, at(w.X, 0, j)))
+      return -4;
+  }
   if (int rc = read_info(w)) return rc;
-  if (rocsolver_dtrtri(w.h, rocblas_fill_upper, rocblas_diagonal_non_unit, n, w.X, n, w.info) !=
-      rocblas_status_success)
-    return -4;
-  if (int rc = read_info(w)) return rc;
-  hipLaunchKernelGGL(k_zero_lower, dim3(grid_nn(nn)), dim3(256), 0, w.st, w.X, n);
-  if (hipGetLastError() != hipSuccess) return -3;
   w.metric_n = n;
   return 0;
 }
