@@ -9,7 +9,7 @@ import ctypes as C
 
 import numpy as np
 
-from .abi import GTOBasis, CONVMETHOD_DIIS4, dptr
+from .abi import GTOBasis, Molecule, CONVMETHOD_DIIS4, dptr
 from .engine import lib
 
 PD = C.POINTER(C.c_double)
@@ -41,8 +41,8 @@ def _bind():
     L.sqscf_density.argtypes = [C.c_void_p, PD, PD]
     L.sqscf_destroy.argtypes = [C.c_void_p]
     L.sqscf_errmsg.restype = C.c_char_p
-    L.sqjk_one_electron.argtypes = [C.c_int, C.POINTER(GTOBasis), C.c_void_p, C.c_int, PD, PD, PD]
-    L.nuclei_coulomb.argtypes = [C.c_void_p]
+    L.sqjk_one_electron.argtypes = [C.c_int, C.POINTER(GTOBasis), C.POINTER(Molecule), C.c_int, PD, PD, PD]
+    L.nuclei_coulomb.argtypes = [C.POINTER(Molecule)]
     L.nuclei_coulomb.restype = C.c_double
     L._scf_bound = True
     return L
@@ -53,7 +53,7 @@ def one_electron(bas, mol):
     L = _bind()
     n = bas.n
     T, V, S = np.zeros((n, n)), np.zeros((n, n)), np.zeros((n, n))
-    rc = L.sqjk_one_electron(n, bas.ptr, C.cast(mol.ptr, C.c_void_p), 0, dptr(T), dptr(V), dptr(S))
+    rc = L.sqjk_one_electron(n, bas.ptr, C.cast(mol.ptr, C.POINTER(Molecule)), 0, dptr(T), dptr(V), dptr(S))
     if rc:
         raise RuntimeError(f"sqjk_one_electron failed ({rc}): {L.sqjk_errmsg().decode()}")
     return T + V, S
@@ -98,7 +98,7 @@ class DeviceSCF:
         p.restricted, p.nEA, p.nEB = int(restricted), nEA, nEB
         p.SCFConv, p.SCFMax, p.SCFDrag = conv, max_iter, drag
         p.threeStep, p.convMethod = int(three_step), method
-        p.Econst = lib().nuclei_coulomb(C.cast(self.mol.ptr, C.c_void_p))
+        p.Econst = lib().nuclei_coulomb(C.cast(self.mol.ptr, C.POINTER(Molecule)))
         p.mixedThreshold = mixed
         r = SCFResult()
         self._check(lib().sqscf_run(self._h, C.byref(p), C.byref(r)), "sqscf_run")
